@@ -118,3 +118,44 @@ def test_long_cached_prefix_beyond_the_staged_page_entries():
     cached prefix (258 pages of 64 over a shuffled table) attend keys on both
     sides of that limit."""
     _prefill_case(70, 4, 2, 64, 0, 0.0, False, 1e4, 1.0, 45, p0=16448)
+
+
+@pytest.mark.parametrize("T,NH,KV,D,window,softcap,p0", [
+    (1, 8, 8, 64, 0, 0.0, 0),         # one row, one head per KV head: a block of 128 positions
+    (129, 4, 4, 128, 0, 50.0, 0),     # a block and one row
+    (65, 8, 1, 128, 31, 0.0, 63),     # 8 heads per KV head, a window inside one key block
+    (17, 8, 2, 256, 0, 0.0, 47),      # one key block, ends with a block's last key
+    (33, 16, 8, 256, 64, 0.0, 64),    # window and prefix on block edges
+    (130, 16, 8, 256, 65, 50.0, 129),
+    (3, 16, 2, 512, 0, 0.0, 29),      # one 32-key block
+    (16, 16, 2, 512, 0, 0.0, 17),     # two 32-key blocks, a whole row block
+    (49, 16, 2, 512, 0, 50.0, 48),    # an odd number of 32-key blocks
+    (96, 16, 2, 512, 0, 50.0, 0),     # the most keys of the few-keys kernel
+    (97, 4, 4, 512, 0, 0.0, 0),       # one more
+    (40, 4, 4, 512, 33, 0.0, 70),
+])
+def test_edges_of_row_and_key_blocks(T, NH, KV, D, window, softcap, p0):
+    """The smallest row and key counts, remainders of the 128-row blocks and of
+    the 32- and 64-key tiles, and each count of query heads per KV head."""
+    _prefill_case(T, NH, KV, D, window, softcap, False, 1e4, 1.0, 46 + T, p0=p0)
+
+
+@pytest.mark.parametrize("D,KV,T", [(64, 2, 200), (256, 8, 200), (512, 2, 90), (512, 2, 150)])
+@pytest.mark.parametrize("page,aligned", [(64, True), (192, False)])
+def test_invalid_pages_read_as_zero(D, KV, T, page, aligned):
+    """A page-table entry outside the pool stands for keys and values of zero
+    (a score of 0): the same bits as with a page of zeros.  With ctx at an
+    address that is not a multiple of 16."""
+    NH, n_pages = 16, (T + page - 1) // page
+    kp, vp = _gen((n_pages + 1, KV, page, D), 60, "kp", 0.3), _gen((n_pages + 1, KV, page, D), 60, "vp")
+    kp[n_pages], vp[n_pages] = 0, 0
+    q = _gen((T, NH, D), 60, "q", 0.3)
+    out = []
+    for bad in (n_pages, -1, n_pages + 5):
+        pt = torch.arange(n_pages, dtype=torch.int32, device=DEV)
+        pt[0] = bad
+        flat = torch.empty(T * NH * D + 1, dtype=torch.bfloat16, device=DEV)
+        ctx = flat[(0 if aligned else 1):][:T * NH * D].view(T, NH, D)
+        out.append(ops.prefill_attention(q, kp, vp, pt, 0, 0, 0.0, ctx=ctx).clone())
+    assert torch.isfinite(out[0].float()).all()
+    assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
