@@ -261,3 +261,70 @@ def test_decode_crosses_the_short_span_graph_boundary(kind):
         if toks_a[i] != toks_b[i]:  # only a near-tie may flip the greedy token
             top2 = torch.topk(b, 2).values
             assert (top2[0] - top2[1]).item() <= 2 * err, f"greedy token differs at position {n0 + i}"
+
+
+def _sample_ref(lg: np.ndarray, top_k: int, t: float, top_p: float, seed: int, step: int) -> int:
+    """The sampler in numpy float32, entry by entry: a stable descending sort of
+    logits / t (ties to the lower index, NaN last), softmax, nucleus cut, one
+    Philox draw."""
+    from oracle.philox import philox4x32_10
+
+    f = np.float32
+    v = lg if t <= 0 else lg / f(max(t, 1e-6))
+    order = np.argsort(np.where(np.isnan(v), f(np.inf), -v), kind="stable")
+    if t <= 0:
+        return int(order[0])
+    k = min(top_k, len(lg))
+    p = np.exp((v[order[:k]] - v[order[0]]).astype(np.float64)).astype(f)
+    z = f(0)
+    for x in p:
+        z = f(z + x)
+    p = (p / z).astype(f)
+    csum, kept = f(0), f(0)
+    for i in range(k):
+        csum = f(csum + p[i])
+        if not f(csum - p[i]) < f(top_p):
+            p[i] = 0
+        kept = f(kept + p[i])
+    u = f(int(philox4x32_10(np.uint32(step), np.uint32(0x53414D50), np.uint32(0), np.uint32(0), seed & 0xFFFFFFFF,
+                            seed >> 32)[0]) >> 8) * f(2.0**-24)
+    acc, last = f(0), 0
+    for i in range(k):
+        if p[i] > 0:
+            last, acc = i, f(acc + p[i])
+            if acc > f(u * kept):
+                break
+    return int(order[last])
+
+
+@pytest.mark.parametrize("V", [1, 3, 63, 257, 4096, 16384, 16385, 65537, 262144, 300001])
+@pytest.mark.parametrize("layout", ["random", "ties", "clustered", "few"])
+def test_sampler_selection_on_every_row_layout(V, layout):
+    """Group counts and sizes at their edges, rows whose largest logits share
+    one group (more candidates than one sort holds), rows of equal logits, rows
+    with a handful of finite ones: the same token as the numpy restatement.  A
+    draw within 1e-5 of a boundary of the cumulative distribution may fall on
+    either side of it (expf against numpy's exp), so the seeds keep clear of
+    those: the kernel's token has to match for each."""
+    rng = np.random.default_rng(V)
+    if layout == "ties":
+        lg = rng.integers(0, 3, V).astype(np.float32)
+    else:
+        lg = (3 * rng.standard_normal(V)).astype(np.float32)
+    if layout == "clustered":  # half of the row, in one stretch, above all the rest
+        lg[V // 4: V // 4 + (V + 1) // 2] += 40.0
+    if layout == "few":
+        keep = rng.permutation(V)[:5]
+        fin = lg[keep].copy()
+        lg[:] = -np.inf
+        lg[keep] = fin
+        if V >= 257:  # (leaves more than 64 entries that are not NaN)
+            lg[rng.permutation(V)[:V // 3]] = np.nan
+        lg[keep[0]] = 1.0
+    dev = torch.from_numpy(lg).to(DEV)
+    tok = torch.zeros(1, dtype=torch.int32, device=DEV)
+    for t, top_k, top_p, seed in ((0.0, 64, 0.9, 1), (1.0, 64, 0.95, 2), (0.7, 5, 1.0, 3), (1.3, 1, 0.5, 2**40 + 4)):
+        ops.sample(dev, top_k, ops.sample_params(t, top_p, seed, DEV), tok, counter_mode=0)
+        if layout == "few" and top_k > 5 and t > 0:
+            top_k = int(np.isfinite(lg).sum())  # masked entries have probability 0
+        assert int(tok.item()) == _sample_ref(lg, top_k, t, top_p, seed, 0), (V, layout, t, top_k)
