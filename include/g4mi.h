@@ -128,7 +128,10 @@ int g4mi_moe_experts_decode(const uint16_t* xn, const uint16_t* gate_up, const u
  * pre_feedforward_layernorm_2 output): router scores, then gate/up with the
  * selection fused in, then down + combine (three kernels); with N > 1 and
  * N*k <= 64 the selection is its own kernel and the gate/up reads a shared
- * expert once (four kernels).  No host sync. */
+ * expert once (four kernels); with N*k > 64 and N <= 64 the experts run grouped
+ * (each selected expert's rows once for all tokens; the same bits) when the
+ * workspace has the size that g4mi_moe_block_workspace_bytes gives.  No host
+ * sync. */
 int64_t g4mi_moe_block_workspace_bytes(int64_t N, int64_t E, int64_t F, int64_t k);
 int g4mi_moe_block_decode(const uint16_t* xn, const uint16_t* router_scale, const uint16_t* router_proj,
                           const uint16_t* per_expert_scale, const uint16_t* gate_up, const uint16_t* down,

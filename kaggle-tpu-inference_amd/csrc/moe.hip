@@ -750,6 +750,20 @@ static int check_experts(const char* what, int64_t N, int64_t H, int64_t F, int6
 
 static inline bool al16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
+// More (token, slot) pairs than one wave's lanes, up to kGroupedTokens tokens:
+// the experts run grouped (prefill.hip: each selected expert's rows stream once
+// for all the tokens that chose it; the same dot products and combine, the same
+// bits).  26B block, router to combine: 9 tokens 146.7 -> 128 us, 16 243.5 ->
+// 172, 32 466 -> 233, 64 912 -> 294; at 8 tokens (64 pairs) the pair kernels,
+// which share repeated rows by a ballot, need two launches less: 107 against 122.
+constexpr int64_t kGroupedTokens = 64;
+static bool grouped_experts(int64_t N, int64_t k) { return N * k > 64 && N <= kGroupedTokens; }
+int moe_experts_grouped(const uint16_t* xn, const float* top_w, const int32_t* top_i, const uint16_t* gate_up,
+                        const uint16_t* down, int64_t n, int64_t H, int64_t F, int64_t E, int64_t K, int32_t combine,
+                        uint16_t* out, void* ws, hipStream_t st);
+
+static int64_t pair_ws_bytes(int64_t N, int64_t F, int64_t k) { return ((N * k * F * 2 + 255) / 256) * 256; }
+
 }  // namespace g4mi
 
 using namespace g4mi;
@@ -827,7 +841,9 @@ int g4mi_moe_down(const uint16_t* act, const uint16_t* down, const int32_t* top_
 }
 
 int64_t g4mi_moe_experts_workspace_bytes(int64_t N, int64_t F, int64_t k) {
-  return ((N * k * F * 2 + 255) / 256) * 256;
+  // (the grouped form's for any H and E that the entry points take)
+  if (grouped_experts(N, k)) return g4mi_moe_prefill_workspace_bytes(N, k, kMaxE, F, 4096);
+  return pair_ws_bytes(N, F, k);
 }
 
 int g4mi_moe_experts_decode(const uint16_t* xn, const uint16_t* gate_up, const uint16_t* down,
@@ -835,9 +851,14 @@ int g4mi_moe_experts_decode(const uint16_t* xn, const uint16_t* gate_up, const u
                             int64_t E, int64_t k, int32_t combine, uint16_t* out, void* ws, int64_t ws_bytes,
                             void* stream) {
   G4MI_REQUIRE(ws != nullptr, G4MI_EINVAL, "moe_experts_decode: null workspace");
-  G4MI_REQUIRE(N >= 1 && k >= 1 && ws_bytes >= g4mi_moe_experts_workspace_bytes(N, F, k), G4MI_EWORKSPACE,
+  G4MI_REQUIRE(N >= 1 && k >= 1 && ws_bytes >= pair_ws_bytes(N, F, k), G4MI_EWORKSPACE,
                "moe_experts_decode: workspace too small");
   G4MI_REQUIRE(al16(ws), G4MI_EALIGN, "moe_experts_decode: workspace must be 16-byte aligned");
+  if (grouped_experts(N, k) && xn && gate_up && down && top_w && top_i && out &&
+      check_experts("moe_experts_decode", N, H, F, E, k) == 0 && al16(xn) && al16(gate_up) && al16(down) &&
+      (combine == G4MI_COMBINE_BF16_RUNNING || combine == G4MI_COMBINE_F32) &&
+      ws_bytes >= g4mi_moe_prefill_workspace_bytes(N, k, E, F, H))  // else as below, or its error
+    return moe_experts_grouped(xn, top_w, top_i, gate_up, down, N, H, F, E, k, combine, out, ws, as_stream(stream));
   uint16_t* act = (uint16_t*)ws;
   int rc = g4mi_moe_gateup(xn, gate_up, top_w, top_i, N, H, F, E, k, act, stream);
   if (rc) return rc;
@@ -853,25 +874,27 @@ int g4mi_moe_block_decode(const uint16_t* xn, const uint16_t* router_scale, cons
                           int64_t N, int64_t H, int64_t F, int64_t E, int64_t k, float eps, int32_t combine,
                           uint16_t* out, float* top_w, int32_t* top_i, void* ws, int64_t ws_bytes, void* stream) {
   G4MI_REQUIRE(ws != nullptr, G4MI_EINVAL, "moe_block_decode: null workspace");
-  G4MI_REQUIRE(N >= 1 && k >= 1 && ws_bytes >= g4mi_moe_block_workspace_bytes(N, E, F, k), G4MI_EWORKSPACE,
+  const int64_t rbytes = g4mi_moe_router_workspace_bytes(N, E);
+  G4MI_REQUIRE(N >= 1 && k >= 1 && ws_bytes >= rbytes + pair_ws_bytes(N, F, k), G4MI_EWORKSPACE,
                "moe_block_decode: workspace too small");
   G4MI_REQUIRE(al16(ws), G4MI_EALIGN, "moe_block_decode: workspace must be 16-byte aligned");
   float* scores = (float*)ws;
-  uint16_t* act = (uint16_t*)((char*)ws + g4mi_moe_router_workspace_bytes(N, E));
+  uint16_t* act = (uint16_t*)((char*)ws + rbytes);
   int rc;
-  if (N > 1 && N * k <= 64) {
-    // several tokens: one selection launch, then the gate/up with the routing
-    // given, which reads an expert chosen by several tokens once
+  if (N > 1 && (N * k <= 64 ||
+                (grouped_experts(N, k) && ws_bytes - rbytes >= g4mi_moe_prefill_workspace_bytes(N, k, E, F, H)))) {
+    // several tokens: one selection launch, then the experts with the routing
+    // given, which read an expert chosen by several tokens once
     rc = g4mi_moe_router_topk(xn, nullptr, router_scale, router_proj, per_expert_scale, N, H, E, k, eps, top_w,
-                              top_i, ws, g4mi_moe_router_workspace_bytes(N, E), stream);
+                              top_i, ws, rbytes, stream);
     if (rc) return rc;
-    rc = g4mi_moe_gateup(xn, gate_up, top_w, top_i, N, H, F, E, k, act, stream);
-  } else {
-    // one token: the selection runs in every gate/up block (no launch between)
-    rc = g4mi_moe_router_scores(xn, nullptr, router_scale, router_proj, N, H, E, eps, scores, stream);
-    if (rc) return rc;
-    rc = g4mi_moe_gateup_routed(xn, scores, per_expert_scale, gate_up, N, H, F, E, k, act, top_w, top_i, stream);
+    return g4mi_moe_experts_decode(xn, gate_up, down, top_w, top_i, N, H, F, E, k, combine, out, act,
+                                   ws_bytes - rbytes, stream);
   }
+  // one token: the selection runs in every gate/up block (no launch between)
+  rc = g4mi_moe_router_scores(xn, nullptr, router_scale, router_proj, N, H, E, eps, scores, stream);
+  if (rc) return rc;
+  rc = g4mi_moe_gateup_routed(xn, scores, per_expert_scale, gate_up, N, H, F, E, k, act, top_w, top_i, stream);
   if (rc) return rc;
   return g4mi_moe_down(act, down, top_i, N, H, F, E, k, combine, out, stream);
 }

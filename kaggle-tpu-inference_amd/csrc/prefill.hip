@@ -613,6 +613,43 @@ static void launch_moe_sort(const int32_t* top_i, const float* top_w, int n, int
                      w.hist, w.a_rows, w.w_sorted, w.slot_pos, w.tiles, w.ntiles, tile_rows);
 }
 
+// The experts of n tokens with their routing, each selected expert's rows read
+// once (the three kernels above and the combine).  H = 256 i, F = 64 j (i, j <=
+// 16), E <= kMaxExperts; ws of g4mi_moe_prefill_workspace_bytes(n, K, E, F, H).
+int moe_experts_grouped(const uint16_t* xn, const float* top_w, const int32_t* top_i, const uint16_t* gate_up,
+                        const uint16_t* down, int64_t n, int64_t H, int64_t F, int64_t E, int64_t K, int32_t combine,
+                        uint16_t* out, void* ws, hipStream_t st) {
+  const MoePrefillWs w = moe_prefill_ws(ws, n, K, E, F, H);
+  // one tile per kTileRows pairs of a selected expert
+  const int tiles = (int)((n * K < E ? n * K : E) + n * K / kTileRows);
+  launch_moe_sort(top_i, top_w, (int)n, (int)K, (int)E, w, kTileRows, st);
+  const dim3 ggrid((unsigned)tiles, (unsigned)((F + 4 * kGrpPairs - 1) / (4 * kGrpPairs)));
+  switch (H / 256) {
+#define G4MI_GU(I)                                                                                             \
+  case I:                                                                                                      \
+    hipLaunchKernelGGL(moe_gateup_grouped_kernel<I>, ggrid, dim3(256), 0, st, xn, gate_up, w.a_rows, w.w_sorted, \
+                       w.tiles, w.ntiles, (int)F, w.act);                                                     \
+    break;
+    G4MI_GU(1) G4MI_GU(2) G4MI_GU(3) G4MI_GU(4) G4MI_GU(5) G4MI_GU(6) G4MI_GU(7) G4MI_GU(8)
+    G4MI_GU(9) G4MI_GU(10) G4MI_GU(11) G4MI_GU(12) G4MI_GU(13) G4MI_GU(14) G4MI_GU(15) G4MI_GU(16)
+#undef G4MI_GU
+  }
+  const dim3 dgrid((unsigned)tiles, (unsigned)((H + 32 * kGrpDownRows - 1) / (32 * kGrpDownRows)));
+  switch (F / 64) {
+#define G4MI_DN(I)                                                                                              \
+  case I:                                                                                                       \
+    hipLaunchKernelGGL(moe_down_grouped_kernel<I>, dgrid, dim3(256), 0, st, w.act, down, w.tiles, w.ntiles,     \
+                       (int)H, w.part);                                                                         \
+    break;
+    G4MI_DN(1) G4MI_DN(2) G4MI_DN(3) G4MI_DN(4) G4MI_DN(5) G4MI_DN(6) G4MI_DN(7) G4MI_DN(8)
+    G4MI_DN(9) G4MI_DN(10) G4MI_DN(11) G4MI_DN(12) G4MI_DN(13) G4MI_DN(14) G4MI_DN(15) G4MI_DN(16)
+#undef G4MI_DN
+  }
+  hipLaunchKernelGGL(moe_combine_kernel, dim3((unsigned)((H / 4 + 255) / 256), (unsigned)n), dim3(256), 0, st, w.part,
+                     w.slot_pos, (int)n, (int)K, (int)H, combine == 0 ? 1 : 0, out);
+  return check_launch("moe experts (grouped)");
+}
+
 }  // namespace g4mi
 
 using namespace g4mi;
@@ -671,37 +708,7 @@ int g4mi_moe_decode_grouped(const uint16_t* xn, const float* top_w, const int32_
                G4MI_EALIGN, "moe_decode_grouped: operands must be 16-byte aligned");
   G4MI_REQUIRE(ws_bytes >= g4mi_moe_prefill_workspace_bytes(n, K, E, F, H), G4MI_EWORKSPACE,
                "moe_decode_grouped: workspace too small (g4mi_moe_prefill_workspace_bytes)");
-  hipStream_t st = as_stream(stream);
-  const MoePrefillWs w = moe_prefill_ws(ws, n, K, E, F, H);
-  // at most n <= 16 pairs per expert: one tile per selected expert
-  const int tiles = (int)(n * K < E ? n * K : E);
-  hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(1024), 0, st, top_i, top_w, (int)n, (int)K, (int)E, w.a_rows,
-                     w.w_sorted, w.slot_pos, w.tiles, w.ntiles, kTileRows);
-  const dim3 ggrid((unsigned)tiles, (unsigned)((F + 4 * kGrpPairs - 1) / (4 * kGrpPairs)));
-  switch (H / 256) {
-#define G4MI_GU(I)                                                                                             \
-  case I:                                                                                                      \
-    hipLaunchKernelGGL(moe_gateup_grouped_kernel<I>, ggrid, dim3(256), 0, st, xn, gate_up, w.a_rows, w.w_sorted, \
-                       w.tiles, w.ntiles, (int)F, w.act);                                                     \
-    break;
-    G4MI_GU(1) G4MI_GU(2) G4MI_GU(3) G4MI_GU(4) G4MI_GU(5) G4MI_GU(6) G4MI_GU(7) G4MI_GU(8)
-    G4MI_GU(9) G4MI_GU(10) G4MI_GU(11) G4MI_GU(12) G4MI_GU(13) G4MI_GU(14) G4MI_GU(15) G4MI_GU(16)
-#undef G4MI_GU
-  }
-  const dim3 dgrid((unsigned)tiles, (unsigned)((H + 32 * kGrpDownRows - 1) / (32 * kGrpDownRows)));
-  switch (F / 64) {
-#define G4MI_DN(I)                                                                                              \
-  case I:                                                                                                       \
-    hipLaunchKernelGGL(moe_down_grouped_kernel<I>, dgrid, dim3(256), 0, st, w.act, down, w.tiles, w.ntiles,     \
-                       (int)H, w.part);                                                                         \
-    break;
-    G4MI_DN(1) G4MI_DN(2) G4MI_DN(3) G4MI_DN(4) G4MI_DN(5) G4MI_DN(6) G4MI_DN(7) G4MI_DN(8)
-    G4MI_DN(9) G4MI_DN(10) G4MI_DN(11) G4MI_DN(12) G4MI_DN(13) G4MI_DN(14) G4MI_DN(15) G4MI_DN(16)
-#undef G4MI_DN
-  }
-  hipLaunchKernelGGL(moe_combine_kernel, dim3((unsigned)((H / 4 + 255) / 256), (unsigned)n), dim3(256), 0, st, w.part,
-                     w.slot_pos, (int)n, (int)K, (int)H, combine == 0 ? 1 : 0, out);
-  return check_launch("moe_decode_grouped");
+  return moe_experts_grouped(xn, top_w, top_i, gate_up, down, n, H, F, E, K, combine, out, ws, as_stream(stream));
 }
 
 int g4mi_rows_embed(const int32_t* tok, int64_t n, const uint16_t* embed, int64_t vocab, const uint16_t* input_ln,

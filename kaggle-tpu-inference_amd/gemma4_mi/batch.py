@@ -175,6 +175,9 @@ class BatchDecodeRunner:
                 if self.grouped_moe and B <= 16:  # each selected expert's rows once for all rows that chose it
                     ops.moe_decode_grouped(self.xe, self.top_w, self.top_i, lp["experts.gate_up_proj"],
                                            lp["experts.down_proj"], "bf16_running", out=self.moe_out)
+                elif self.grouped_moe:  # more than 16 rows: grouped too, inside the library
+                    ops.moe_experts(self.xe, lp["experts.gate_up_proj"], lp["experts.down_proj"], self.top_w,
+                                    self.top_i, "bf16_running", out=self.moe_out)
                 else:
                     ops.moe_gateup(self.xe, lp["experts.gate_up_proj"], self.top_w, self.top_i, act=self.act_moe)
                     ops.moe_down(self.act_moe, lp["experts.down_proj"], self.top_i, "bf16_running", out=self.moe_out)

@@ -419,3 +419,43 @@ def test_wave_selection_equals_block_selection(e, k, n):
     print(f"E={e} k={k}: {tied} of {n} rows hold tied scores")
     assert torch.equal(ti_b, ti_w)
     assert torch.equal(tw_b.view(torch.int32), tw_w.view(torch.int32))
+
+
+@pytest.mark.parametrize("N", [9, 17, 33, 64, 65])
+@pytest.mark.parametrize("E,K,H,F", [(16, 8, 256, 128), (128, 8, 2816, 704)])
+@pytest.mark.parametrize("combine", ["bf16_running", "f32"])
+def test_experts_of_many_tokens_equal_the_pair_kernels(N, E, K, H, F, combine):
+    """More than 64 (token, slot) pairs: the grouped form (up to 64 tokens), or
+    the pair kernels where the workspace is smaller than the grouped form needs,
+    give the gate/up and down pair kernels' bits; an expert index outside [0, E)
+    counts as a routing weight of 0; a token may name an expert twice."""
+    g = torch.Generator(device=DEV).manual_seed(N + E)
+    r = lambda *s, std=1.0: torch.empty(s, dtype=torch.bfloat16, device=DEV).normal_(0, std, generator=g)  # noqa: E731
+    xn, gu, dn = r(N, H), r(E, 2, F, H, std=0.05), r(E, H, F, std=0.05)
+    top_w = torch.rand((N, K), device=DEV, generator=g)
+    top_i = torch.randint(0, E, (N, K), device=DEV, dtype=torch.int32, generator=g)
+    top_i[0, 1], top_i[N - 1, 0] = E, -1
+    top_i[:, 2] = 3  # one expert of every token
+    exp = ops.moe_down(ops.moe_gateup(xn, gu, top_w, top_i), dn, top_i, combine)
+    got = ops.moe_experts(xn, gu, dn, top_w, top_i, combine)
+    assert torch.equal(got, exp)
+    small = torch.empty((N * K * F * 2 + 255) // 256 * 256, dtype=torch.uint8, device=DEV)
+    out = torch.empty_like(exp)
+    p = ops._ptr
+    ops._lib.call("g4mi_moe_experts_decode", p(xn), p(gu), p(dn), p(top_w), p(top_i), N, H, F, E, K,
+                  {"bf16_running": 0, "f32": 1}[combine], p(out), p(small), small.numel(), ops.stream_handle())
+    assert torch.equal(out, exp)
+
+
+@pytest.mark.parametrize("N", [8, 9, 16, 40, 65])
+def test_moe_block_of_many_tokens_equals_its_parts(N):
+    """The block at 26B widths, across the token counts where its route changes."""
+    H, E, K, F = 2816, 128, 8, 704
+    g = torch.Generator(device=DEV).manual_seed(N)
+    r = lambda *s, std=1.0, mean=0.0: torch.empty(s, dtype=torch.bfloat16, device=DEV).normal_(mean, std, generator=g)  # noqa: E731
+    xn, sc, pr, pes = r(N, H), r(H, std=0.1, mean=1.0), r(E, H, std=2.0), r(E, std=0.1, mean=1.0)
+    gu, dn = r(E, 2, F, H, std=0.02), r(E, H, F, std=0.02)
+    out, tw, ti = ops.moe_block(xn, sc, pr, pes, gu, dn, K, 1e-6)
+    ew, ei = ops.moe_router_topk(xn, sc, pr, pes, K, 1e-6)
+    assert torch.equal(ti, ei) and torch.equal(tw, ew)
+    assert torch.equal(out, ops.moe_down(ops.moe_gateup(xn, gu, ew, ei), dn, ei))
