@@ -523,100 +523,104 @@ static float bf16_inv_sqrt(int64_t H) {
 
 // Many rows (prefill) on f64 MFMA (v_mfma_f64_16x16x4_f64: lane l supplies
 // A[l%16][l/16] and B[l/16][l%16] and holds D[4r + l/16][l%16], r < 4).  A
-// block takes kRouterMRows = 16 token rows and 64 experts: the rows are
-// normalised into LDS (the same rounding steps as router_scores_kernel),
-// then wave w accumulates the 16 x 16 dots of experts 64*blockIdx.y + 16w ..
-// +15 in f64 (the bf16 x bf16 products are exact; the sum is f64 as in the
-// per-row kernels, in another order).  Per 32-wide k chunk lane l reads 8
-// consecutive k of row l%16 (LDS) and of expert l%16 (router row, 16 bytes)
-// at chunk offset 8*(l/16), and MFMA s of the chunk takes k = 8*(l/16) + s:
-// the four k slots of the MFMA cover the chunk over s = 0..7.  H % 32 == 0,
+// block of 16 waves takes kRouterMRows = 16 token rows and 64 experts: wave w
+// normalises row w into LDS (the same rounding steps as router_scores_kernel),
+// then waves (eg = w % 4, kq = w / 4) accumulate the 16 x 16 dots of experts
+// 64*blockIdx.y + 16 eg .. +15 over the kq-th quarter of K in f64 (the bf16 x
+// bf16 products are exact; the sum is f64 as in the per-row kernels, in another
+// order), and the parts are added in order through LDS.  Per 32-wide k chunk
+// lane l reads 8 consecutive k of row l%16 (LDS) and of expert l%16 (router row,
+// 16 bytes) at chunk offset 8*(l/16), and MFMA s of the chunk takes k = 8*(l/16)
+// + s: the four k slots of the MFMA cover the chunk over s = 0..7.  H % 32 == 0,
 // H <= kRouterMaxH.
+// The f64 MFMAs are the bound from 2,048 rows on (1.5 GFLOP in 36 us with every
+// SIMD busy); below, too few blocks: EG is the largest of 4, 2, 1 that leaves at
+// least 192.  LDS rows are padded by one 16-byte slot, so that the 16 rows of a
+// fragment read (5,632 bytes apart at H = 2,816) spread over the banks.
+// 26B router, 128 / 500 / 1,000 / 2,048 / 4,096 rows: 42.6 / 43.6 / 43.9 / 45.0 /
+// 86.0 -> 16.4 / 17.0 / 22.6 / 36.6 / 71.5 us (before: 64 experts per block, 4
+// waves with 4 rows to normalise and the whole K each; 127 rows on the per-row
+// kernel: 14.0).
 constexpr int kRouterMRows = 16;
-constexpr int kRouterMExperts = 64;
 constexpr int kRouterMaxH = 4096;
 typedef double f64x4 __attribute__((ext_vector_type(4)));
-__global__ __launch_bounds__(256) void router_scores_mfma_kernel(const uint16_t* __restrict__ x,
-                                                                 const uint16_t* __restrict__ pre_w,
-                                                                 const uint16_t* __restrict__ scale,
-                                                                 const uint16_t* __restrict__ proj, int N, int H,
-                                                                 int E, float eps, float inv_sqrt_h_bf,
-                                                                 float* __restrict__ scores) {
-  __shared__ u32x4 xs_rows[kRouterMRows * kRouterMaxH / 8];  // 16 x H/8 chunks
+template <int EG>
+__global__ __launch_bounds__(1024) void router_scores_mfma_kernel(const uint16_t* __restrict__ x,
+                                                                  const uint16_t* __restrict__ pre_w,
+                                                                  const uint16_t* __restrict__ scale,
+                                                                  const uint16_t* __restrict__ proj, int N, int H,
+                                                                  int E, float eps, float inv_sqrt_h_bf,
+                                                                  float* __restrict__ scores) {
+  constexpr int KQ = 16 / EG;                                      // parts of K
+  __shared__ u32x4 xs_rows[kRouterMRows * (kRouterMaxH / 8 + 1)];  // 16 rows of H/8 chunks and one of padding
+  __shared__ double part[KQ - 1][EG][4][64];                       // parts 1 .. of K: [kq - 1][eg][r][lane]
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
   const int CH = H / 8;
   const int r0 = blockIdx.x * kRouterMRows;
-  const int e0 = blockIdx.y * kRouterMExperts + wave * 16;
-  const u32x4* pw = (const u32x4*)pre_w;
-  const u32x4* sw = (const u32x4*)scale;
+  const int eg = wave % EG, kq = wave / EG;
+  const int e0 = (blockIdx.y * EG + eg) * 16;
+  const int nch = CH / 4, c0 = nch * kq / KQ, c1 = nch * (kq + 1) / KQ;  // this wave's 32-wide k chunks
   // this wave's first router rows, requested before the normalisation
   const int er = min(e0 + (lane & 15), E - 1);
   const u32x4* wrow = (const u32x4*)(proj + (size_t)er * H) + (lane >> 4);
-  constexpr int PF = 8;  // router chunks in flight per lane
+  constexpr int PF = 4;  // router chunks in flight per lane
   u32x4 wq[PF];
 #pragma unroll
-  for (int u = 0; u < PF; ++u) wq[u] = ld16(wrow + 4 * min(u, CH / 4 - 1));
-  // the wave's 4 token rows and both norm weights, all requested at once
-  // (one round trip, not three per row), then normalised from registers
-  constexpr int RW = kRouterMRows / 4;                 // rows per wave
-  constexpr int XPL = (kRouterMaxH / 8 + 63) / 64;     // 16-byte chunks per lane and row
-  u32x4 xv[RW][XPL], pwv[XPL], scv[XPL];
+  for (int u = 0; u < PF; ++u) wq[u] = ld16(wrow + 4 * min(c0 + u, nch - 1));
+  {
+    // row r0 + wave, from registers; the norm weights follow chunk by chunk
+    constexpr int XPL = (kRouterMaxH / 8 + 63) / 64;  // 16-byte chunks per lane
+    u32x4 v[XPL];
+    const u32x4* xr = (const u32x4*)(x + (size_t)min(r0 + wave, N - 1) * H);
+    const u32x4* pw = (const u32x4*)(pre_w != nullptr ? pre_w : scale);
+    const u32x4* sw = (const u32x4*)scale;
 #pragma unroll
-  for (int j = 0; j < XPL; ++j) {
-    const int cc = min(lane + 64 * j, CH - 1);
-    pwv[j] = ld16((pre_w != nullptr ? pw : sw) + cc);
-    scv[j] = ld16(sw + cc);
-#pragma unroll
-    for (int rr = 0; rr < RW; ++rr) {
-      const int r = wave * RW + rr;
-      xv[rr][j] = ld16((const u32x4*)(x + (size_t)min(r0 + r, N - 1) * H) + cc);
-    }
-  }
-#pragma unroll
-  for (int rr = 0; rr < RW; ++rr) {
-    const int r = wave * RW + rr;
-    float rp = 1.0f;
+    for (int j = 0; j < XPL; ++j)
+      if (64 * j < CH) v[j] = ld16(xr + min(lane + 64 * j, CH - 1));
     if (pre_w != nullptr) {  // pre_feedforward_layernorm_2 (model.py:315)
       double s0 = 0.0;
 #pragma unroll
       for (int j = 0; j < XPL; ++j)
-        if (lane + 64 * j < CH) s0 = sumsq8_f64(xv[rr][j], s0);
-      rp = rms_scale(group_sum_f64<64>(s0), H, eps);
+        if (lane + 64 * j < CH) s0 = sumsq8_f64(v[j], s0);
+      const float rp = rms_scale(group_sum_f64<64>(s0), H, eps);
 #pragma unroll
-      for (int j = 0; j < XPL; ++j) xv[rr][j] = scale8(xv[rr][j], rp, &pwv[j]);
+      for (int j = 0; j < XPL; ++j)
+        if (64 * j < CH) {
+          const u32x4 pj = ld16(pw + min(lane + 64 * j, CH - 1));
+          v[j] = scale8(v[j], rp, &pj);
+        }
     }
     double s1 = 0.0;
 #pragma unroll
     for (int j = 0; j < XPL; ++j)
-      if (lane + 64 * j < CH) s1 = sumsq8_f64(xv[rr][j], s1);
+      if (lane + 64 * j < CH) s1 = sumsq8_f64(v[j], s1);
     const float r1 = rms_scale(group_sum_f64<64>(s1), H, eps);
 #pragma unroll
     for (int j = 0; j < XPL; ++j) {
       const int c8 = lane + 64 * j;
       if (c8 < CH) {
+        const u32x4 sc = ld16(sw + c8);
         float f[8], g[8];
-        unpack8(xv[rr][j], f);
-        unpack8(scv[j], g);
+        unpack8(v[j], f);
+        unpack8(sc, g);
 #pragma unroll
         for (int q = 0; q < 8; ++q) f[q] = rbf(rbf(rbf(f[q] * r1) * g[q]) * inv_sqrt_h_bf);
         u32x4 o;
         o.x = pack2(f[0], f[1]); o.y = pack2(f[2], f[3]); o.z = pack2(f[4], f[5]); o.w = pack2(f[6], f[7]);
-        xs_rows[r * CH + c8] = o;
+        xs_rows[wave * (CH + 1) + c8] = o;
       }
     }
   }
   __syncthreads();
-  if (e0 >= E) return;  // no barrier below
-  const u32x4* xrow = xs_rows + (lane & 15) * CH + (lane >> 4);
+  const u32x4* xrow = xs_rows + (lane & 15) * (CH + 1) + (lane >> 4);
   // two accumulator chains (even and odd k slots of each MFMA group), so
   // consecutive MFMAs do not wait for each other's result; summed at the end
   f64x4 acc[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
-  const int nch = CH / 4;  // 32-wide k chunks
-  for (int c0 = 0; c0 < nch; c0 += PF) {
+  for (int cb = c0; cb < c1; cb += PF) {
 #pragma unroll
     for (int u = 0; u < PF; ++u) {
-      const int c = c0 + u;
-      if (c < nch) {
+      const int c = cb + u;
+      if (c < c1) {
         const u32x4 wv = wq[u];
         wq[u] = ld16(wrow + 4 * min(c + PF, nch - 1));  // chunk c + PF (clamped: a cache hit at the end)
         const u32x4 xv = xrow[4 * c];
@@ -630,11 +634,20 @@ __global__ __launch_bounds__(256) void router_scores_mfma_kernel(const uint16_t*
       }
     }
   }
+  if (kq > 0) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) part[kq - 1][eg][r][lane] = acc[0][r] + acc[1][r];
+  }
+  __syncthreads();
+  if (kq > 0) return;
   const int e = e0 + (lane & 15);
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int n = r0 + 4 * r + (lane >> 4);
-    if (n < N && e < E) scores[(size_t)n * E + e] = rbf(f32_of(acc[0][r] + acc[1][r]));
+    double d = acc[0][r] + acc[1][r];
+#pragma unroll
+    for (int q = 0; q < KQ - 1; ++q) d += part[q][eg][r][lane];
+    if (n < N && e < E) scores[(size_t)n * E + e] = rbf(f32_of(d));
   }
 }
 
@@ -646,10 +659,14 @@ static void launch_scores(const uint16_t* x, const uint16_t* pre_w, const uint16
   // (~5 us at 54 rows, ~200 us at 2,048)
   if (N >= 128 && H % 32 == 0 && H <= kRouterMaxH && ((uintptr_t)scale & 15u) == 0 &&
       ((uintptr_t)pre_w & 15u) == 0) {
-    const dim3 tgrid((unsigned)((N + kRouterMRows - 1) / kRouterMRows),
-                     (unsigned)((E + kRouterMExperts - 1) / kRouterMExperts));
-    hipLaunchKernelGGL(router_scores_mfma_kernel, tgrid, dim3(256), 0, st, x, pre_w, scale, proj, N, H, E, eps, c,
-                       scores);
+    const int rows = (N + kRouterMRows - 1) / kRouterMRows;
+#define G4MI_ROUTER(G)                                                                                          \
+  hipLaunchKernelGGL(router_scores_mfma_kernel<G>, dim3((unsigned)rows, (unsigned)((E + 16 * G - 1) / (16 * G))), \
+                     dim3(1024), 0, st, x, pre_w, scale, proj, N, H, E, eps, c, scores)
+    if (rows * ((E + 63) / 64) >= 192) G4MI_ROUTER(4);
+    else if (rows * ((E + 31) / 32) >= 192) G4MI_ROUTER(2);
+    else G4MI_ROUTER(1);
+#undef G4MI_ROUTER
     return;
   }
   const bool aligned = ((uintptr_t)scale & 15u) == 0 && ((uintptr_t)pre_w & 15u) == 0;

@@ -459,3 +459,19 @@ def test_moe_block_of_many_tokens_equals_its_parts(N):
     ew, ei = ops.moe_router_topk(xn, sc, pr, pes, K, 1e-6)
     assert torch.equal(ti, ei) and torch.equal(tw, ew)
     assert torch.equal(out, ops.moe_down(ops.moe_gateup(xn, gu, ew, ei), dn, ei))
+
+
+@pytest.mark.parametrize("N", [128, 143, 1000, 2100, 3100])
+@pytest.mark.parametrize("E,H", [(16, 256), (72, 800), (128, 2816), (200, 4096)])
+def test_router_scores_of_many_rows_equal_the_row_kernels(N, E, H):
+    """Every split of experts and K over a block of the many-rows kernel gives
+    the scores of the kernels for fewer rows, bit for bit, with and without the
+    pre-norm."""
+    g = torch.Generator(device=DEV).manual_seed(N + E)
+    r = lambda *s, std=1.0, mean=0.0: torch.empty(s, dtype=torch.bfloat16, device=DEV).normal_(mean, std, generator=g)  # noqa: E731
+    x, sc, pr, pn = r(N, H), r(H, std=0.1, mean=1.0), r(E, H, std=0.5), r(H, std=0.1, mean=1.0)
+    for pre in (None, pn):
+        got = ops.moe_router_scores(x, sc, pr, 1e-6, pre_norm_w=pre)
+        exp = torch.cat([ops.moe_router_scores(x[i:i + 100].contiguous(), sc, pr, 1e-6, pre_norm_w=pre)
+                         for i in range(0, N, 100)])
+        assert torch.equal(got, exp)
