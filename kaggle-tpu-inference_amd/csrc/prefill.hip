@@ -564,14 +564,26 @@ static float bf16_round_host(double v) {
   return f;
 }
 
-// Expert tile height: 192 rows while the experts average 96 to 176 rows (an
-// expert's rows then mostly spill past 128 but fit 192, and every further
-// tile of an expert streams its weights again), else 128.
+// Tiles an expert of x rows takes on average, x ~ N(a, a) (even routing), at h
+// rows per tile: the sum over j of P(x > j h).
+static double tiles_per_expert(double a, int h) {
+  double t = 0.0;
+  for (int j = 0; j * (double)h < a + 6.0 * sqrt(a); ++j) t += 0.5 * erfc((j * (double)h - a) / sqrt(2.0 * a));
+  return t;
+}
+
+// Expert tile height: every further tile of an expert streams its weights again,
+// so 192 rows where that leaves fewer tiles, else 128 (whose blocks are shorter);
+// from 96 rows per expert on, below that nearly every expert is one tile of
+// either.  26B block, us at 128 / 192: 2,048 tokens (128 rows per expert) 574 /
+// 475, 2,816 (176) 796 / 615, 3,077 (192) 814 / 733, 3,600 (225: two tiles of
+// either) 864 / 881, 4,096 (256) 1,022 / 908.
 // G4MI_MOE_TILE_ROWS = 128 or 192 overrides.
 static int moe_prefill_tile_rows(int64_t pairs, int64_t E) {
   const char* e = getenv("G4MI_MOE_TILE_ROWS");
   if (e != nullptr && (atoi(e) == 128 || atoi(e) == 192)) return atoi(e);
-  return (pairs >= 96 * E && pairs < 176 * E) ? 192 : 128;
+  const double a = (double)pairs / (double)E;
+  return (a >= 96.0 && tiles_per_expert(a, 192) < 0.98 * tiles_per_expert(a, 128)) ? 192 : 128;
 }
 
 struct MoePrefillWs {
