@@ -352,3 +352,31 @@ def test_rows_tail_experts_equals_combine_then_tail(which, n):
     torch.cuda.synchronize()
     assert torch.equal(xa.view(torch.int16), xb.view(torch.int16))
     assert torch.equal(xna.view(torch.int16), xnb.view(torch.int16))
+
+
+@pytest.mark.parametrize("M,N,K", [(17, 128, 64), (65, 130, 128), (300, 201, 192), (130, 1028, 704)])
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("slices", [1, 2])
+def test_gemm_output_rows_of_any_alignment(M, N, K, f32, slices):
+    """The 16-byte stores of whole patches, their last columns, and the
+    element-wise stores of rows that are not 16-byte aligned: the same values
+    wherever the output lies, and nothing outside it."""
+    slices = min(slices, K // 64)
+    g = torch.Generator(device=DEV).manual_seed(M)
+    a = torch.empty((M, K), dtype=torch.bfloat16, device=DEV).normal_(generator=g)
+    b = torch.empty((N, K), dtype=torch.bfloat16, device=DEV).normal_(generator=g)
+    ep = ops.EP_F32 if f32 else ops.EP_BF16
+    dt = torch.float32 if f32 else torch.bfloat16
+    ref = (a.double() @ b.double().T)
+    outs = []
+    for pad, off in ((0, 0), (1, 0), (8, 0), (8, 3)):
+        buf = torch.full((M * (N + pad) + 64,), 7.0, dtype=dt, device=DEV)
+        out = buf[off:off + M * (N + pad)].view(M, N + pad)
+        ops.gemm(a, b, out=out, epilogue=ep, n=N, k_slices=slices, ldc=N + pad)
+        assert (out[:, N:] == 7.0).all() and (buf[:off] == 7.0).all() and (buf[off + M * (N + pad):] == 7.0).all()
+        outs.append(out[:, :N].clone())
+    for o in outs:
+        assert torch.equal(o, outs[0])
+    # f32 sums of K products: within K * 2^-24 of the magnitudes' sum; bf16: half an ulp more
+    tol = (a.double().abs() @ b.double().abs().T) * K * 2.0**-24 + (0 if f32 else ref.abs() * 2.0**-8)
+    assert ((outs[0].double() - ref).abs() <= tol).all()
