@@ -635,6 +635,27 @@ int g4mi_gemm_bf16(const uint16_t* a, int64_t lda, const int32_t* a_rows, const 
 
 namespace g4mi {
 
+// Whether a plain product of M rows takes 192-row tiles rather than its
+// `tiles` 128-row ones.  The 256 CUs hold 512 blocks at a time, and what counts
+// is how many such rounds the tiles need and how full the last one is: at
+// K = 2,816 a round of two 128-row blocks per CU takes 43 us and one of at
+// most one block per CU 30; with 192 rows 56 us and 37-45 (K = 2,112 and 4,096
+// in the same proportions), hence 10, 7, 13 and 10 below.  Measured either
+// side of the line, 128 rows against 192: gate/up of 2,000 rows (528 tiles or
+// 363) 73.9 us against 55.8, of 1,900 rows (495 or 330) 45.2 against 55.9, of
+// 3,072 rows (792 or 528) 81.5 against 95.4; 8,192 columns at 1,100 rows 68.1
+// against 49.8, at 2,048 rows 86.8 against 89.9, at 4,096 rows 200.7 against
+// 165.3; 2,816 columns over 4,096 inputs at 2,800 rows 59.3 against 67.5, at
+// 3,072 rows 93.7 against 68.5.
+static bool tall_tiles(int64_t M, int64_t tiles) {
+  const int64_t tall = tiles / ((M + 127) / 128) * ((M + 191) / 192);
+  const auto cost = [](int64_t n, int64_t full, int64_t half) {
+    const int64_t rest = n % 512;
+    return n / 512 * full + (rest == 0 ? 0 : rest <= 256 ? half : full);
+  };
+  return cost(tall, 13, 10) < cost(tiles, 10, 7);
+}
+
 // g4mi_gemm_bf16 with grouped tiles of up to tile_rows (128 or 192) rows: the
 // MoE prefill's expert tiles are 192 rows once most experts have more than
 // 128 rows (one tile per expert, so its weights stream once, still two
@@ -692,10 +713,11 @@ int gemm_bf16_tiles(const uint16_t* a, int64_t lda, const int32_t* a_rows, const
   }
   // grouped tiles are up to 128 rows (128-row kernels) or, through
   // gemm_bf16_tiles, 192; small plain M takes
-  // 64-row tiles.  Two blocks per CU (2 stages) for grouped tiles and when
-  // there are more tiles than CUs, else one block per CU with 3 stages.
+  // 64-row tiles, and a plain product takes 192-row ones where tall_tiles
+  // says so.  Two blocks per CU (2 stages) for grouped tiles, 192-row ones and
+  // when there are more tiles than CUs, else one block per CU with 3 stages.
   const bool small = tiles == nullptr && M <= 64;
-  const int64_t mtiles = tiles ? max_tiles : (M + (small ? 63 : 127)) / (small ? 64 : 128);
+  int64_t mtiles = tiles ? max_tiles : (M + (small ? 63 : 127)) / (small ? 64 : 128);
   const int64_t ncol = epilogue == kEpGated ? 64 : 128;
   const int64_t nblocks = mtiles * ((N + ncol - 1) / ncol) * k_slices;
   G4MI_REQUIRE(mtiles * ((N + ncol - 1) / ncol) <= 2147483647 - 8, G4MI_EINVAL, "gemm: too many tiles");
@@ -707,7 +729,8 @@ int gemm_bf16_tiles(const uint16_t* a, int64_t lda, const int32_t* a_rows, const
   else launch<BM, BN, S, O, kEpBf16>(g, mtiles, st);
   if (small) {
     G4MI_GEMM(64, 128, 3, 1)
-  } else if (tiles != nullptr && tile_rows == 192) {
+  } else if (tiles != nullptr ? tile_rows == 192 : k_slices == 1 && tall_tiles(M, nblocks)) {
+    if (tiles == nullptr) mtiles = (M + 191) / 192;
     G4MI_GEMM(192, 128, 2, 2)
   } else if (tiles != nullptr || nblocks > 256) {
     G4MI_GEMM(128, 128, 2, 2)

@@ -165,6 +165,30 @@ def test_gemm_prefill_shapes(m, n, k):
     _check_f32(out32, ref, absum)
 
 
+@pytest.mark.parametrize("m,n", [(513, 13120), (577, 13120), (1025, 7300), (1153, 8192), (768, 16300)])
+def test_gemm_tall_tiles(m, n):
+    """Plain products of a little more than 512 128-row tiles take 192-row
+    ones: one row into a tile, a whole number of tiles, ragged columns; each
+    of their rows equals the same row among so few that 128-row tiles run."""
+    k = 320
+    a, b = _rand((m, k), 31), _rand((n, k), 32, 0.02)
+    ref, absum = _ref(a, b)
+    ad, bd = a.to(DEV), b.to(DEV)
+    out = ops.gemm(ad, bd)
+    _check_bf16(out, ref, absum)
+    _check_f32(ops.gemm(ad, bd, epilogue=ops.EP_F32), ref, absum)
+    cut = 256
+    for i in range(0, m, cut):
+        few = ops.gemm(ad[i:i + cut], bd[:2048])
+        assert torch.equal(few.view(torch.int16), out[i:i + cut, :2048].contiguous().view(torch.int16))
+    rows = torch.tensor(np.random.default_rng(5).integers(0, m, size=m), dtype=torch.int32)
+    got = ops.gemm(ad, bd, a_rows=rows.to(DEV))
+    assert torch.equal(got.view(torch.int16), out[rows.long().to(DEV)].view(torch.int16))
+    half = n // 2
+    gated = ops.gemm(ad, bd, epilogue=ops.EP_GATED, pair_offset=half * k, n=half)
+    _close_bf16(gated, _gated_ref(a, b[:half], b[half:2 * half], None))
+
+
 @pytest.mark.parametrize("m", [17, 300, 2048])
 def test_prefill_gemm_gated_separate_tensors(m):
     """The dense MLP's gate/up product as the prefill issues it: gate and up
