@@ -184,9 +184,11 @@ __device__ __forceinline__ void norm_rope_slice(float* x, const float* w, const 
 // nothing to prefetch.  NW = 8 (long ranges): 8 waves, each owning tiles w
 // and w + 8 of a split's 16 at most, all requested by the end of the q
 // prologue (part of the first before it, see KS0), so a whole split's K rows
-// are in flight at once.
-template <int D, int G, bool ONE, int NW, bool DPT>
-__global__ __launch_bounds__(NW * 64) void attn_qk_kernel(
+// are in flight at once.  OCC = 2 (8 waves): half the registers, so that two
+// blocks share a CU: the q fragments are read from LDS at each step and the
+// second tile's chunks take the registers of the first's as they are used.
+template <int D, int G, bool ONE, int NW, bool DPT, int OCC = 1>
+__global__ __launch_bounds__(NW * 64, OCC * NW / 4) void attn_qk_kernel(
     AttnDims a, const uint16_t* __restrict__ q_raw, const uint16_t* __restrict__ k_raw,
     const uint16_t* __restrict__ v_raw, const uint16_t* __restrict__ q_norm, const uint16_t* __restrict__ k_norm,
     const uint16_t* __restrict__ rope_cos, const uint16_t* __restrict__ rope_sin, uint16_t* __restrict__ k_pages,
@@ -196,9 +198,10 @@ __global__ __launch_bounds__(NW * 64) void attn_qk_kernel(
   constexpr int NT = NW * 64;
   constexpr int GW = (G + NW - 1) / NW;
   constexpr int KS = D / 32;  // MFMA steps along the head dimension
-  constexpr int TPW = (NW == 8 && !ONE) ? kChunkMax / 16 / NW : 1;  // tiles requested up front per wave
+  constexpr int TPW = (NW == 8 && !ONE && OCC == 1) ? kChunkMax / 16 / NW : 1;  // tiles requested up front per wave
+  constexpr int QS = D + 8;  // an LDS row of q: 16 rows' chunks start in different banks
   static_assert(NW == 4 || NW == 8, "4 or 8 waves");
-  __shared__ __align__(16) uint16_t qa[16 * D];
+  __shared__ __align__(16) uint16_t qa[16 * QS];
   __shared__ __align__(16) uint16_t kn16[D];
   __shared__ float knew[D];
   __shared__ float vnew[D];
@@ -278,14 +281,14 @@ __global__ __launch_bounds__(NW * 64) void attn_qk_kernel(
   constexpr int KS0 = (NW == 8 && KS > 8) ? 8 : KS;
   load_chunks(0, 0, KS0);
   // padding rows G..15 of the A operand are zero
-  for (int c = tid; c < (16 - G) * D / 8; c += NT) ((u32x4*)(qa + G * D))[c] = u32x4{0u, 0u, 0u, 0u};
+  for (int c = tid; c < (16 - G) * QS / 8; c += NT) ((u32x4*)(qa + G * QS))[c] = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
   for (int u = 0; u < GW; ++u) {
     const int g = wave + NW * u;
     if (g < G) {
       norm_rope_slice<D>(qx[u], qw, cs, sn, a.eps, true);
 #pragma unroll
-      for (int i = 0; i < PL; ++i) qa[g * D + so + i] = f2bf(qx[u][i]);
+      for (int i = 0; i < PL; ++i) qa[g * QS + so + i] = f2bf(qx[u][i]);
     }
   }
   if (mine && wave >= 2) {
@@ -311,12 +314,15 @@ __global__ __launch_bounds__(NW * 64) void attn_qk_kernel(
       }
   }
 
-  u32x4 af[KS];
+  auto qfrag = [&](int s) { return *(const u32x4*)(qa + col * QS + 32 * s + 8 * kg); };
+  u32x4 af[OCC == 1 ? KS : 1];
+  if constexpr (OCC == 1) {
 #pragma unroll
-  for (int s = 0; s < KS; ++s) af[s] = *(const u32x4*)(qa + col * D + 32 * s + 8 * kg);
+    for (int s = 0; s < KS; ++s) af[s] = qfrag(s);
+  }
   const float cap = a.softcap;
   // scores of tile t (K rows in bf) into sc
-  auto score_tile = [&](int t, const u32x4* bf, long long off) {
+  auto score_tile = [&](int t, u32x4* bf, long long off, auto refill) {
     const int j = t * 16 + col;
     const bool isnew = mine && (start + j == pos);
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -324,8 +330,9 @@ __global__ __launch_bounds__(NW * 64) void attn_qk_kernel(
     for (int s = 0; s < KS; ++s) {
       u32x4 kb = bf[s];
       if (mine) kb = isnew ? *(const u32x4*)(kn16 + 32 * s + 8 * kg) : kb;
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, af[s]), __builtin_bit_cast(bf16x8, kb),
-                                                    acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, OCC == 1 ? af[s] : qfrag(s)),
+                                                    __builtin_bit_cast(bf16x8, kb), acc, 0, 0, 0);
+      refill(s);
     }
     const bool ok = (off >= 0) || isnew;
 #pragma unroll
@@ -338,12 +345,22 @@ __global__ __launch_bounds__(NW * 64) void attn_qk_kernel(
       }
     }
   };
+  const auto keep = [](int) {};
   if constexpr (ONE) {
-    if (wave < ntiles) score_tile(wave, bt[0], ot[0]);
+    if (wave < ntiles) score_tile(wave, bt[0], ot[0], keep);
+  } else if constexpr (NW == 8 && OCC == 2) {
+    // the wave's second tile takes the registers of the first chunk by chunk
+    // (clamped to the split, so a wave without one reads rows it may read)
+    const int j1 = min(min(wave + NW, ntiles - 1) * 16 + col, npos - 1);
+    const long long o1 = page_off_lds(a, ptl, first, start + j1, kv);
+    const uint16_t* kp1 = k_pages + max(o1, 0ll) + 8 * kg;
+    if (wave < ntiles)
+      score_tile(wave, bt[0], ot[0], [&](int s) { bt[0][s] = ld16((const u32x4*)(kp1 + 32 * s)); });
+    if (wave + NW < ntiles) score_tile(wave + NW, bt[0], o1, keep);
   } else if constexpr (NW == 8) {
 #pragma unroll
     for (int tt = 0; tt < TPW; ++tt)
-      if (wave + NW * tt < ntiles) score_tile(wave + NW * tt, bt[tt], ot[tt]);
+      if (wave + NW * tt < ntiles) score_tile(wave + NW * tt, bt[tt], ot[tt], keep);
   } else {
     u32x4 bcur[KS];
 #pragma unroll
@@ -355,7 +372,7 @@ __global__ __launch_bounds__(NW * 64) void attn_qk_kernel(
       // the next tile of this wave, or this tile again on the last pass (a
       // cache hit, so the barrier after the loop does not wait on HBM)
       load_tile(t + 4 < ntiles ? t + 4 : t, bnext, onext);
-      score_tile(t, bcur, ocur);
+      score_tile(t, bcur, ocur, keep);
 #pragma unroll
       for (int s = 0; s < KS; ++s) bcur[s] = bnext[s];
       ocur = onext;
@@ -628,8 +645,12 @@ __device__ __forceinline__ void pv_short(const AttnDims& a, const Range& R, int 
 // Writes the wave's partial sums to v_out (per head, 8 dims per lane, summed
 // over the PPV positions of a step).
 constexpr int kPvRing = 12;
+// With two blocks per CU: P.V of eight sequences of 2,000 to 8,191 positions
+// (head_dim 512) 34.8 us with 4, 36.2 with 6, 37.2 with 8, and 38.9 with one
+// block per CU.
+constexpr int kPvRing2 = 4;
 
-template <int D, int G, typename PT>
+template <int D, int G, int RING, typename PT>
 __device__ __forceinline__ void pv_long8(const AttnDims& a, const Range& R, int split, int kv, int b,
                                          const uint16_t* __restrict__ v_pages, const PT& pt_row,
                                          const float* ws_scores, const float* ws_stats,
@@ -640,7 +661,7 @@ __device__ __forceinline__ void pv_long8(const AttnDims& a, const Range& R, int 
   constexpr int LPV = DW / 8;                   // lanes per position
   constexpr int PPV = 64 / LPV;                 // positions per wave step
   constexpr int MAXST = kChunkMax / PPV;        // steps per split at most
-  constexpr int RB = kPvRing < MAXST ? kPvRing : MAXST;  // steps in flight
+  constexpr int RB = RING < MAXST ? RING : MAXST;  // steps in flight
   constexpr int RB0 = RB < 8 ? RB : 8;                   // of which requested before the merge
   constexpr int RS = (G * kChunkMax + NT - 1) / NT;  // scores per thread
   static_assert(D % (NW * 8) == 0 && MAXST % 2 == 0 && RB % 2 == 0, "pv_long8 layout");
@@ -748,8 +769,8 @@ __device__ __forceinline__ void pv_long8(const AttnDims& a, const Range& R, int 
   slot_out = slot;
 }
 
-template <int D, int G, int NW, bool DPT>
-__global__ __launch_bounds__(NW * 64) void attn_pv_kernel(AttnDims a, const uint16_t* __restrict__ v_pages,
+template <int D, int G, int NW, bool DPT, int OCC = 1>
+__global__ __launch_bounds__(NW * 64, OCC * NW / 4) void attn_pv_kernel(AttnDims a, const uint16_t* __restrict__ v_pages,
                                                       const int32_t* __restrict__ page_table,
                                                       const int32_t* __restrict__ pos_arr,
                                                       const float* ws_scores,
@@ -790,8 +811,8 @@ __global__ __launch_bounds__(NW * 64) void attn_pv_kernel(AttnDims a, const uint
   if constexpr (NW == 8) {
     float v[G][8];
     int dofs, slot;
-    pv_long8<D, G>(a, R, split, kv, b, v_pages, pt_row_of<DPT>(a, page_table, b), ws_scores, ws_stats, lds_f, mg,
-                   sg, ptl, v, dofs, slot);
+    pv_long8<D, G, OCC == 2 ? kPvRing2 : kPvRing>(a, R, split, kv, b, v_pages, pt_row_of<DPT>(a, page_table, b),
+                                                  ws_scores, ws_stats, lds_f, mg, sg, ptl, v, dofs, slot);
     // the partials are reduced by attn_reduce_kernel, the next launch
     if (slot == 0) {
 #pragma unroll
@@ -1427,10 +1448,22 @@ static void launch_attn(const AttnDims& a, dim3 grid, hipStream_t st, const uint
     hipLaunchKernelGGL((attn_pv_kernel<D, G, 4, DPT>), pgrid, dim3(256), 0, st, a, vp, pt, pos, w.scores, w.stats,
                        w.part, w.group, w.counters, ctx);
   } else {
-    hipLaunchKernelGGL((attn_qk_kernel<D, G, false, 8, DPT>), grid, dim3(512), 0, st, a, q_raw, k_raw, v_raw,
-                       q_norm, k_norm, cs, sn, kp, vp, pt, pos, append, w.scores, w.stats);
-    hipLaunchKernelGGL((attn_pv_kernel<D, G, 8, DPT>), pgrid, dim3(512), 0, st, a, vp, pt, pos, w.scores, w.stats,
-                       w.part, w.group, w.counters, ctx);
+    // More blocks than the 256 CUs (several sequences): two blocks per CU, so
+    // one block's start and softmax run behind the other's rows.  Eight
+    // sequences of 2,000 to 8,191 positions (544 blocks), two KV heads
+    // of 512 with 8 query heads each: qk 31.8 -> 25.0 us, P.V 39 -> 35.  Up to 256 blocks there
+    // is one block per CU anyway, and it requests its whole split at once.
+    if ((int64_t)grid.x * grid.y * grid.z > 256) {
+      hipLaunchKernelGGL((attn_qk_kernel<D, G, false, 8, DPT, 2>), grid, dim3(512), 0, st, a, q_raw, k_raw, v_raw,
+                         q_norm, k_norm, cs, sn, kp, vp, pt, pos, append, w.scores, w.stats);
+      hipLaunchKernelGGL((attn_pv_kernel<D, G, 8, DPT, 2>), pgrid, dim3(512), 0, st, a, vp, pt, pos, w.scores,
+                         w.stats, w.part, w.group, w.counters, ctx);
+    } else {
+      hipLaunchKernelGGL((attn_qk_kernel<D, G, false, 8, DPT>), grid, dim3(512), 0, st, a, q_raw, k_raw, v_raw,
+                         q_norm, k_norm, cs, sn, kp, vp, pt, pos, append, w.scores, w.stats);
+      hipLaunchKernelGGL((attn_pv_kernel<D, G, 8, DPT>), pgrid, dim3(512), 0, st, a, vp, pt, pos, w.scores, w.stats,
+                         w.part, w.group, w.counters, ctx);
+    }
     const dim3 rgrid((unsigned)((G * D / 4 + kRedCols - 1) / kRedCols), grid.y, grid.z);
     hipLaunchKernelGGL((attn_reduce_kernel<D, G>), rgrid, dim3(256), 0, st, a, pos, w.part, ctx);
   }

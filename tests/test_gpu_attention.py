@@ -339,3 +339,33 @@ def test_dense_page_table_needs_enough_pages():
                       ops._ptr(cos), ops._ptr(cos), ops._ptr(kp), ops._ptr(kp), 3, None, ops_max_pages,
                       ops._ptr(pos), 2, 4, 2, 64, 16, 0, 0.0, 1e-6, 1, 64, 1, ops._ptr(ctx), ops._ptr(ws), ws.numel(),
                       ops.stream_handle(q.device))
+
+
+@pytest.mark.parametrize("kv,d,window", [(2, 512, 0), (4, 256, 0), (4, 256, 4200)])
+def test_many_long_sequences_equal_each_alone(kv, d, window):
+    """More than 256 blocks over long ranges (8-wave blocks, two per CU)
+    against each sequence in a call of its own (at most 256 blocks, one per
+    CU), the same split count in both: outputs and appended rows are the same
+    bits.  Lengths either side of 512, of one tile per wave, of the smallest
+    split times the count, the last position, and a position outside."""
+    nh, page, lmax, splits = kv * 8 if d == 512 else kv * 2, 64, 17 * 256, 17
+    lens = [513, 600, 17 * 64, 17 * 64 + 1, 17 * 128 + 5, lmax - 1, lmax, 0]
+    b, mp = len(lens), lmax // page
+    assert b * kv * splits > 256 >= kv * splits
+    q, k, v = _gen((b, nh, d), 41, "q"), _gen((b, kv, d), 41, "k"), _gen((b, kv, d), 41, "v")
+    qn, kn = _gen((d,), 41, "qn", 0.5), _gen((d,), 41, "kn", 0.5)
+    cos, sin = gm.rope_table(d, 1e4, 1.0, lmax, DEV)
+    kp, vp = _gen((b * mp, kv, page, d), 41, "kp"), _gen((b * mp, kv, page, d), 41, "vp")
+    pt = torch.randperm(b * mp, generator=torch.Generator().manual_seed(41)).to(torch.int32).reshape(b, mp)
+    pt[1, 3] = -1
+    pt = pt.to(DEV)
+    pos = torch.tensor([n - 1 for n in lens], dtype=torch.int32, device=DEV)
+    ka, va = kp.clone(), vp.clone()
+    got = ops.decode_attention(q, k, v, qn, kn, cos, sin, ka, va, pt, pos, window, 0.0, 1e-6, lmax, n_split_max=splits)
+    for i in range(b):
+        one = ops.decode_attention(q[i:i + 1], k[i:i + 1], v[i:i + 1], qn, kn, cos, sin, kp, vp, pt[i:i + 1],
+                                   pos[i:i + 1], window, 0.0, 1e-6, lmax, n_split_max=splits)
+        assert torch.equal(got[i].view(torch.int16), one[0].view(torch.int16)), lens[i]
+    assert torch.equal(ka.view(torch.int16), kp.view(torch.int16)) and torch.equal(va.view(torch.int16),
+                                                                                  vp.view(torch.int16))
+    assert not bool(got[-1].any())
