@@ -42,10 +42,10 @@
 // measured on random operands).
 //
 // Measured (26B-A4B layers, us, before = 16 rows per wave on 16x16x32 with V
-// transposed by 2-byte LDS stores): full layer, 4,096 rows: 1,271 -> 424;
-// sliding layer, 2,000 rows: 125 -> 60.  At 4,096 rows a 32-key block costs a
-// wave 8.0 kcycles of which 96 MFMAs are 4.3; what bounds it is the issue of
-// the ~1,000 other instructions of a wave that is alone on its SIMD.
+// transposed by 2-byte LDS stores): full layer, 4,096 rows: 1,268 -> 414;
+// sliding layer, 2,000 rows: 125 -> 63.  At 4,096 rows a 32-key block costs a
+// wave 6.9 kcycles of which its 96 MFMAs are 4.3; what bounds the rest is the
+// issue of the other instructions of a wave that is alone on its SIMD.
 #include <math.h>
 
 #include "capi_util.h"
